@@ -61,10 +61,13 @@ struct GemmPlan {
     int panel;       // > 0: column-panel kernel (2: level tables staged in LDS)
     int panel_stages;  // column-panel ring depth
     int panel_waves;   // column-panel waves per workgroup
+    int wide_cols, wide_chunks;  // wide_chunks > 0: wide kernel, column blocks x row chunks
 };
 
 #ifdef CUBIC_EXPERIMENTS
 // experiment builds only: force the panel plan (J, split, tables in LDS)
+static int g_wide = 0;  // 1: wide kernel, -1: never
+extern "C" __attribute__((visibility("default"))) void cubic_exp_wide(int w, int) { g_wide = w; }
 static int g_exp_j = 0, g_exp_split = 0, g_exp_tl = -1, g_exp_panel = -1, g_exp_stages = 0, g_exp_waves = 0;
 extern "C" __attribute__((visibility("default"))) void cubic_exp_plan(int j, int split, int tl, int panel, int stages, int waves) {
     g_exp_j = j; g_exp_split = split; g_exp_tl = tl; g_exp_panel = panel; g_exp_stages = stages; g_exp_waves = waves;
@@ -125,6 +128,70 @@ void plan_k(int64_t n_member, int64_t k, int bits, int* split_out, int* bps_out)
     *split_out = (int)ceil_div(k_blocks, bps);
 }
 
+// MFMA-tile kernel (gemm_kernel): tiles per wave and rows per workgroup.
+void plan_tiles_per_wave(int64_t m, int group_in, GemmPlan* p) {
+    // Past 64 rows (whole-k-block groups) a workgroup takes 128 rows: each
+    // decoded weight fragment feeds eight m-tiles of MFMA instead of four.
+    const bool wide = m > 64 && group_in % kKBlock == 0;
+    const int64_t chunks = ceil_div(m, wide ? 128 : 64);
+    // Two 16-column tiles per wave (half the activation bytes and A-fragment
+    // LDS reads per weight byte) when K is whole and the launch still fills the
+    // GPU; one tile per wave otherwise.
+    p->tiles_per_wave = (p->split == 1 && ceil_div(p->n_tiles, 2 * cubic::kGemmWaves) * chunks >= 256) ? 2 : 1;
+    // Past 64 rows the A-fragment LDS reads bound the loop (one MFMA per
+    // fragment at J = 1): two tiles per wave whenever the grid keeps >= 320
+    // workgroups (Llama-3-70B layers at M = 65..512: 12-25% faster per layer;
+    // a narrower grid, o at M <= 128, measured slower).
+    if (wide && ceil_div(p->n_tiles, 2 * cubic::kGemmWaves) * p->split * chunks >= 320) p->tiles_per_wave = 2;
+    p->col_blocks = (int)ceil_div(p->n_tiles, cubic::kGemmWaves * p->tiles_per_wave);
+    // Rows 33..64 split over two 32-row workgroups when the grid would
+    // otherwise hold fewer than two workgroups per CU (qkv, o: measured 7%
+    // faster; the weights are read twice, from L2 the second time).
+    p->chunk_rows = wide ? 128 : 64;
+    if (p->tiles_per_wave == 1 && m > 32 && m <= 64 && (int64_t)p->col_blocks * p->split < 512)
+        p->chunk_rows = 32;
+}
+
+// Wide kernel (cubic_wide.hip) instead of the MFMA-tile plan in *p, by the time
+// either is expected to take (us), fitted to launches of M = 200 to 2048 over
+// 2048, 4096 and 8192-wide layers at 4 bits (within about 10% of them):
+//   wide: rounds of 256 workgroups (one per CU), 2.0 per k-block;
+//   MFMA tiles: rounds of 512 workgroups, 2.3 per k-block (two tiles per wave;
+//     64-row chunks, for groups below a k-block, 1.7, and 0.85 with one tile),
+//     a last round of up to 128 workgroups at half, up to 5 a round where
+//     partitions are too short to hide their first loads, and the K split's
+//     partials, written and read at 6.7 TB/s (of two only one is stored).
+// The wide kernel wins where its 256 x 128 tiles fill their rounds (us, MFMA
+// tiles against wide: 4096 -> 2 x 12288 M = 256 78 / 64, 1024 247 / 206, 2048
+// 487 / 408; 4096 -> 6144 M = 1024 89 / 64; 12288 -> 4096 M = 2048 282 / 195;
+// 2048 -> 2 x 6144 M = 512 65 / 39) and loses where they leave CUs idle that
+// K partitions would use (12288 -> 4096 M = 1024, 128 workgroups, 149 / 164;
+// M = 512 88 / 163; 4096 -> 6144 M = 512 53 / 60).
+void plan_wide(int64_t m, int bits, GemmPlan* p) {
+    // one tile per wave over 128-row chunks: fewer than 320 workgroups of two,
+    // never enough for wide tiles
+    if (bits > 4 || m <= 64 || (p->chunk_rows == 128 && p->tiles_per_wave == 1)) return;
+    const int64_t cols = ceil_div((int64_t)p->n_tiles * 16, cubic::kWideCols);
+    const int64_t chunks = ceil_div(m, cubic::kWideRows);
+    if (cols * chunks >= (int64_t(1) << 31)) return;
+    const double wide = 2.0 + (double)ceil_div(cols * chunks, 256) * p->k_blocks * 2.0;
+    const int64_t blocks = (int64_t)p->col_blocks * ceil_div(m, p->chunk_rows);
+    const int64_t wgs = blocks * p->split, rest = wgs % 512;
+    const double rounds = (double)(wgs / 512) + (rest == 0 ? 0.0 : rest <= 128 ? 0.5 : 1.0);
+    const double step = p->chunk_rows == 128 ? 2.3 : p->tiles_per_wave == 2 ? 1.7 : 0.85;
+    const double start = p->split > 1 && p->blocks_per_split < 7 ? 7.0 - p->blocks_per_split : 0.0;
+    const double stored = p->split == 1 ? 0.0 : p->split == 2 ? 1.0 : (double)p->split;
+    const double block_bytes = 8.0 * p->chunk_rows * (16 * cubic::kGemmWaves * p->tiles_per_wave);
+    const double tiles = rounds * (p->blocks_per_split * step + start) + stored * (double)blocks * block_bytes / 6.7e6;
+    bool take = wide < tiles;
+#ifdef CUBIC_EXPERIMENTS
+    if (g_wide) take = g_wide > 0;
+#endif
+    if (!take) return;
+    p->wide_cols = (int)cols;
+    p->wide_chunks = (int)chunks;
+}
+
 GemmPlan plan_gemm(int64_t m, int64_t n_member, int members, int64_t k, int bits, int group_in) {
     GemmPlan p = {};
     const int64_t n = n_member * members;
@@ -179,26 +246,8 @@ GemmPlan plan_gemm(int64_t m, int64_t n_member, int members, int64_t k, int bits
             return p;
         }
     }
-    // Past 64 rows (whole-k-block groups) a workgroup takes 128 rows: each
-    // decoded weight fragment feeds eight m-tiles of MFMA instead of four.
-    const bool wide = m > 64 && group_in % kKBlock == 0;
-    const int64_t chunks = ceil_div(m, wide ? 128 : 64);
-    // Two 16-column tiles per wave (half the activation bytes and A-fragment
-    // LDS reads per weight byte) when K is whole and the launch still fills the
-    // GPU; one tile per wave otherwise.
-    p.tiles_per_wave = (p.split == 1 && ceil_div(p.n_tiles, 2 * cubic::kGemmWaves) * chunks >= 256) ? 2 : 1;
-    // Past 64 rows the A-fragment LDS reads bound the loop (one MFMA per
-    // fragment at J = 1): two tiles per wave whenever the grid keeps >= 320
-    // workgroups (Llama-3-70B layers at M = 65..512: 12-25% faster per layer;
-    // a narrower grid, o at M <= 128, measured slower).
-    if (wide && ceil_div(p.n_tiles, 2 * cubic::kGemmWaves) * p.split * chunks >= 320) p.tiles_per_wave = 2;
-    p.col_blocks = (int)ceil_div(p.n_tiles, cubic::kGemmWaves * p.tiles_per_wave);
-    // Rows 33..64 split over two 32-row workgroups when the grid would
-    // otherwise hold fewer than two workgroups per CU (qkv, o: measured 7%
-    // faster; the weights are read twice, from L2 the second time).
-    p.chunk_rows = wide ? 128 : 64;
-    if (p.tiles_per_wave == 1 && m > 32 && m <= 64 && (int64_t)p.col_blocks * p.split < 512)
-        p.chunk_rows = 32;
+    plan_tiles_per_wave(m, group_in, &p);
+    plan_wide(m, bits, &p);
     return p;
 }
 
@@ -207,7 +256,7 @@ GemmPlan plan_gemm(int64_t m, int64_t n_member, int members, int64_t k, int bits
 // tiles x MT m-tiles x 64 lanes float4 units.
 int64_t gemm_workspace(int64_t m, int64_t n_member, int members, int64_t k, int bits, int group_in) {
     const GemmPlan p = plan_gemm(m, n_member, members, k, bits, group_in);
-    if (p.split == 1) return 0;
+    if (p.split == 1 || p.wide_chunks) return 0;
     const int64_t blocks = (int64_t)p.col_blocks * ceil_div(m, p.chunk_rows);
     const int64_t mt = p.chunk_rows == 128 ? 8 : p.chunk_rows == 32 ? 2 : (ceil_div(m, 64) > 1 ? 4 : (m >= 33 ? 4 : (m >= 17 ? 2 : 1)));
     const int64_t units = (p.panel ? p.panel_waves : cubic::kGemmWaves) *
@@ -263,6 +312,17 @@ int gemm_common(const void* x, int64_t ldx, const uint32_t* codes, const uint32_
                                 align256((int64_t)p.split * p.col_blocks * cubic::kGemmWaves * 4 * 64 * 16);
         if (workspace_bytes < alt) return fail(CUBIC_EWORKSPACE, "gemm workspace %lld < %lld bytes", (long long)workspace_bytes, (long long)alt);
     }
+    if (p.wide_chunks && (ldx >= (int64_t(1) << 28) || ceil_div(k, group_in) * 256 >= (int64_t(1) << 31))) {
+        // the wide kernel's 32-bit offsets span four rows, and a tile's
+        // metadata: extents this large take the MFMA-tile kernel (same K plan,
+        // same arithmetic)
+        p.wide_chunks = 0;
+        const int64_t blocks = (int64_t)p.col_blocks * ceil_div(m, p.chunk_rows);
+        const int64_t alt = p.split == 1 ? 0
+                          : align256(blocks * 4) + align256((int64_t)p.split * blocks * cubic::kGemmWaves * p.tiles_per_wave * (p.chunk_rows / 16) * 64 * 16);
+        if (workspace_bytes < alt) return fail(CUBIC_EWORKSPACE, "gemm workspace %lld < %lld bytes", (long long)workspace_bytes, (long long)alt);
+        if (alt && !workspace) return fail(CUBIC_EINVAL, "null workspace");
+    }
     if (need && !workspace) return fail(CUBIC_EINVAL, "null workspace");
     cubic::GemmArgs a = {};
     a.x = (const uint16_t*)x;
@@ -290,8 +350,10 @@ int gemm_common(const void* x, int64_t ldx, const uint32_t* codes, const uint32_
     a.panel = p.panel;
     a.panel_stages = p.panel_stages;
     a.panel_waves = p.panel_waves;
+    a.wide_cols = p.wide_cols;
+    a.wide_chunks = p.wide_chunks;
     a.f16 = dtype == CUBIC_DTYPE_F16;
-    if (p.split > 1) {
+    if (p.split > 1 && workspace) {
         const int64_t counters = align256((int64_t)p.col_blocks * ceil_div(m, p.chunk_rows) * 4);  // one per output block
         a.counters = (uint32_t*)workspace;
         a.partials = (float*)((char*)workspace + counters);

@@ -13,6 +13,9 @@ namespace cubic {
 // workgroups measured slower on every cfg2 shape.
 constexpr int kGemmWaves = 4;
 
+// Wide GEMM workgroup: rows x columns (cubic_wide.hip).
+constexpr int kWideRows = 256, kWideCols = 128;
+
 // Members of one grouped GEMM launch (same K, same per-member width).
 constexpr int kMaxGemmMembers = 8;
 
@@ -156,6 +159,7 @@ struct GemmArgs {
     int panel;                    // > 0: column-panel kernel (2: level tables staged in LDS)
     int panel_stages;             // column-panel ring depth S (2 or 4; divides the partition's k-block pairs)
     int panel_waves;              // column-panel waves per workgroup (the kernels take 4)
+    int wide_cols, wide_chunks;   // wide_chunks > 0: wide kernel, column blocks x row chunks
     // routed experts (MoE, routed != 0): workgroup chunk z covers the
     // 16 * MT padded route slots [z * 16 * MT, ...) of one expert
     // (block_expert[z]); a slot holds a route ordinal, or `routes` for
@@ -263,6 +267,8 @@ hipError_t launch_prepare(const void* packed, const float* scale, const uint16_t
 hipError_t launch_gemm(const GemmArgs& a, hipStream_t s);
 // Column-panel kernel (cubic_panel.hip), chosen by the host plan (a.panel > 0).
 hipError_t launch_panel_gemm(const GemmArgs& a, hipStream_t s);
+// Wide kernel (cubic_wide.hip), chosen by the host plan (a.wide_chunks > 0).
+hipError_t launch_wide_gemm(const GemmArgs& a, hipStream_t s);
 // Routed-block table from compact routes (quantization/common/marlin/repack.py:253-277)
 hipError_t launch_pad_routes(const int32_t* counts, const int32_t* starts, const int32_t* block_starts,
                              const int32_t* total_blocks, const int32_t* row_map, int experts,

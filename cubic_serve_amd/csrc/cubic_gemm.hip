@@ -744,6 +744,7 @@ hipError_t launch_gemm(const GemmArgs& a, hipStream_t s) {
             default: return hipErrorInvalidValue;
         }
     }
+    if (a.wide_chunks) return launch_wide_gemm(a, s);  // host plan: prompt-sized M, bits <= 4
     if (a.panel) return launch_panel_gemm(a, s);  // host plan: M <= 64, bits <= 4, whole-k-block groups
     // routed: one grid chunk per padded route block (a.m = block capacity)
     const int mt = a.routed ? a.block_m / 16 : (a.m >= 33 ? 4 : (a.m >= 17 ? 2 : 1));
