@@ -37,8 +37,19 @@ typedef __attribute__((ext_vector_type(8))) _Float16 f16x8_t;
 // accumulates in FP32 (ops/eager/quantization.py:181-186).
 template <bool F16>
 __device__ __forceinline__ uint32_t pack_level2(float lo, float hi) {
-    if constexpr (F16) return float_to_f16_bits(lo) | (float_to_f16_bits(hi) << 16);
-    else return pack_bf16x2(lo, hi);
+    if constexpr (F16) {
+        // one conversion of the two (round to nearest even); the pins keep a
+        // producing multiply from being folded into it (one rounding where
+        // the reference makes two)
+        asm("" : "+v"(lo));
+        asm("" : "+v"(hi));
+        typedef __attribute__((ext_vector_type(2))) _Float16 half2_t;
+        typedef __attribute__((ext_vector_type(2))) float float2_t;
+        const float2_t f = {lo, hi};
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, half2_t));
+    } else {
+        return pack_bf16x2(lo, hi);
+    }
 }
 
 template <bool F16>
