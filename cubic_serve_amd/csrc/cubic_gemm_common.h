@@ -22,10 +22,13 @@ constexpr int kKBlock = 128;
 // (lanes 0..15 store rows 0..15 of one chunk) in position r ^ g(c): both run at
 // the b128 peak rate of gfx950's LDS (measured 243 B/clk/CU for the reads,
 // 83 B/clk/CU for the writes; the plain r ^ c swizzle reads at 128).
-// bf16 per activation stage of a workgroup with MT m-tiles (at least 64 rows:
-// the output tile of the epilogue reuses the stages)
+// bf16 per activation stage of a workgroup with MT m-tiles (the output tile
+// of the epilogue fits two stages at every MT).  Stages of 64 rows whatever
+// MT held 32 KB of LDS for 8 KB of activations and set the workgroups per CU
+// of wide launches at M <= 16 and above 4 bits: Llama-3-70B gate/up at M = 8
+// 138 -> 128 us at 6 bits, 161 -> 147 at 8.
 template <int MT>
-__host__ __device__ constexpr int a_stage() { return (MT > 4 ? MT : 4) * 16 * kKBlock; }
+__host__ __device__ constexpr int a_stage() { return MT * 16 * kKBlock; }
 __device__ __forceinline__ int a_slot(int r16, int c) { return c * 16 + (r16 ^ ((c & 3) << 2) ^ (c >> 2)); }
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
