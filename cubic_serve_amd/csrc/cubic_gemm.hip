@@ -268,7 +268,7 @@ void gemm_kernel(GemmArgs a) {
                     else if constexpr (LT)
                         bw = table_fragment<BITS>(codes[j], f, &lv_lds[((wave * J + j) * 16 + col) * NMP]);
                     else
-                        bw = direct_fragment<BITS, F16>(codes[j], f, ms[j], ma[j], mb[j], t_lds);
+                        bw = direct_fragment<BITS, F16, true>(codes[j], f, ms[j], ma[j], mb[j], t_lds);
 #pragma unroll
                     for (int mt = 0; mt < MT; ++mt)
                         acc[mt][j] = mfma16<F16>(__builtin_bit_cast(uint4, afrag_buf[fb][mt]), bw, acc[mt][j]);
@@ -475,7 +475,7 @@ __global__ __launch_bounds__(64 * G) void rows_kernel(GemmArgs a) {
                 uint4 bw;
                 if constexpr (BITS <= 4) bw = decode_fragment<BITS>(rc[st], f, tab);
                 else if constexpr (LT) bw = table_fragment<BITS>(rc[st], f, lv);
-                else bw = direct_fragment<BITS, F16>(rc[st], f, ms, ma, mb, t_lds);
+                else bw = direct_fragment<BITS, F16, false>(rc[st], f, ms, ma, mb, t_lds);
                 acc = mfma16<F16>(afrag(ra[st], f), bw, acc);
             }
         }
