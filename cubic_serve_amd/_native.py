@@ -29,6 +29,7 @@ SIGNATURES: dict[str, tuple] = {
     "cubic_gemm_workspace_bytes": (I64, [I64, I64, I64, I32]),
     "cubic_gemm_group_workspace_bytes": (I64, [I64, I32, I64, I64, I32]),
     "cubic_gemm_grouped_workspace_bytes": (I64, [I64, I64, I64, I64, I32]),
+    "cubic_gemm_launch_plan": (I64, [I64, I32, I64, I64, I32, I32, I64, P, P]),
     "cubic_gemm_group": (I32, [P, I64, P, P, I64, I32, I64, I64, I32, I32, I32, P, P, P, I64, P]),
     "cubic_gemm": (I32, [P, I64, P, P, I64, I64, I64, I32, I32, I32, P, I64, P, I64, P]),
     "cubic_gemm_grouped": (I32, [P, I64, P, P, I64, I64, I64, I64, I32, I32, I32, P, I64, P, I64, P,

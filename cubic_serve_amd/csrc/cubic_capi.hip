@@ -251,17 +251,24 @@ GemmPlan plan_gemm(int64_t m, int64_t n_member, int members, int64_t k, int bits
     return p;
 }
 
-// Split-K workspace: arrival counters per output block, then FP32 partials
-// per K partition and output block (64-row chunk x column block): waves x J
-// tiles x MT m-tiles x 64 lanes float4 units.
-int64_t gemm_workspace(int64_t m, int64_t n_member, int members, int64_t k, int bits, int group_in) {
-    const GemmPlan p = plan_gemm(m, n_member, members, k, bits, group_in);
-    if (p.split == 1 || p.wide_chunks) return 0;
+// Split-K workspace of the plan's MFMA-tile or column-panel kernel: arrival
+// counters per output block, then FP32 partials per K partition and output
+// block (64-row chunk x column block): waves x J tiles x MT m-tiles x 64 lanes
+// float4 units.
+int64_t split_workspace(const GemmPlan& p, int64_t m) {
+    if (p.split == 1) return 0;
     const int64_t blocks = (int64_t)p.col_blocks * ceil_div(m, p.chunk_rows);
     const int64_t mt = p.chunk_rows == 128 ? 8 : p.chunk_rows == 32 ? 2 : (ceil_div(m, 64) > 1 ? 4 : (m >= 33 ? 4 : (m >= 17 ? 2 : 1)));
     const int64_t units = (p.panel ? p.panel_waves : cubic::kGemmWaves) *
                           p.tiles_per_wave * mt * 64;
     return align256(blocks * 4) + align256((int64_t)p.split * blocks * units * 16);
+}
+
+// The size query: what the split-K kernels need at this m, also where the wide
+// kernel (which needs none) is planned.  It then covers every smaller m of the
+// matrix, and the launches of this m that cannot take the wide kernel.
+int64_t gemm_workspace(int64_t m, int64_t n_member, int members, int64_t k, int bits, int group_in) {
+    return split_workspace(plan_gemm(m, n_member, members, k, bits, group_in), m);
 }
 
 // Workspace when the group width is not known yet: the larger of the two
@@ -271,6 +278,28 @@ int64_t gemm_workspace_any_group(int64_t m, int64_t n_member, int members, int64
     const int64_t b = gemm_workspace(m, n_member, members, k, bits, 32);
     return a > b ? a : b;
 }
+
+// The plan of one launch, the activation row stride known: extents that the
+// 32-bit offsets of the column-panel kernel (all rows) or of the wide kernel
+// (four rows, and a tile's metadata) do not span take the MFMA-tile kernel
+// (same K plan, same arithmetic; its split-K buffer is no larger than the
+// column-panel kernel's).
+GemmPlan plan_launch(int64_t m, int64_t n_member, int members, int64_t k, int bits, int group_in, int64_t ldx) {
+    GemmPlan p = plan_gemm(m, n_member, members, k, bits, group_in);
+    if (p.panel && m * ldx * 2 >= (int64_t(1) << 31)) {
+        p.panel = 0;
+        p.tiles_per_wave = 1;
+        p.col_blocks = (int)ceil_div(p.n_tiles, cubic::kGemmWaves);
+        p.chunk_rows = 64;
+    }
+    if (p.wide_chunks && (ldx >= (int64_t(1) << 28) || ceil_div(k, group_in) * 256 >= (int64_t(1) << 31)))
+        p.wide_chunks = 0;
+    return p;
+}
+
+// What the launch itself needs: nothing where the wide kernel folds the K
+// partitions in registers.
+int64_t launch_workspace(const GemmPlan& p, int64_t m) { return p.wide_chunks ? 0 : split_workspace(p, m); }
 
 int gemm_common(const void* x, int64_t ldx, const uint32_t* codes, const uint32_t* meta,
                 int64_t m, int members, int64_t n_member, int64_t k, int bits, int group_in, int dtype,
@@ -293,36 +322,12 @@ int gemm_common(const void* x, int64_t ldx, const uint32_t* codes, const uint32_
         return fail(CUBIC_ENOTSUP, "activations need k %% 8 == 0, ldx %% 8 == 0 and 16-byte alignment");
     for (int i = 0; i < members; ++i)
         if (ldys[i] < n_member) return fail(CUBIC_EINVAL, "output leading dimension too small");
-    GemmPlan p = plan_gemm(m, n_member, members, k, bits, group_in);
-    const int64_t need = gemm_workspace(m, n_member, members, k, bits, group_in);
-    if (workspace_bytes < need) return fail(CUBIC_EWORKSPACE, "gemm workspace %lld < %lld bytes", (long long)workspace_bytes, (long long)need);
+    const GemmPlan p = plan_launch(m, n_member, members, k, bits, group_in, ldx);
     if (p.rows_waves && m * ldx * 2 >= (int64_t(1) << 31))
         return fail(CUBIC_ENOTSUP, "small-row GEMM: activation row stride too large (m * ldx * 2 = %lld >= 2^31 bytes)",
                     (long long)(m * ldx * 2));
-    if (p.panel && m * ldx * 2 >= (int64_t(1) << 31)) {
-        // the column-panel kernel reaches activations through 32-bit buffer
-        // offsets: a row stride this large takes the MFMA-tile kernel (same
-        // K plan, same arithmetic), whose split-K buffer is no larger
-        p.panel = 0;
-        p.tiles_per_wave = 1;
-        p.col_blocks = (int)ceil_div(p.n_tiles, cubic::kGemmWaves);
-        p.chunk_rows = 64;
-        const int64_t alt = p.split == 1 ? 0
-                          : align256((int64_t)p.col_blocks * 4) +
-                                align256((int64_t)p.split * p.col_blocks * cubic::kGemmWaves * 4 * 64 * 16);
-        if (workspace_bytes < alt) return fail(CUBIC_EWORKSPACE, "gemm workspace %lld < %lld bytes", (long long)workspace_bytes, (long long)alt);
-    }
-    if (p.wide_chunks && (ldx >= (int64_t(1) << 28) || ceil_div(k, group_in) * 256 >= (int64_t(1) << 31))) {
-        // the wide kernel's 32-bit offsets span four rows, and a tile's
-        // metadata: extents this large take the MFMA-tile kernel (same K plan,
-        // same arithmetic)
-        p.wide_chunks = 0;
-        const int64_t blocks = (int64_t)p.col_blocks * ceil_div(m, p.chunk_rows);
-        const int64_t alt = p.split == 1 ? 0
-                          : align256(blocks * 4) + align256((int64_t)p.split * blocks * cubic::kGemmWaves * p.tiles_per_wave * (p.chunk_rows / 16) * 64 * 16);
-        if (workspace_bytes < alt) return fail(CUBIC_EWORKSPACE, "gemm workspace %lld < %lld bytes", (long long)workspace_bytes, (long long)alt);
-        if (alt && !workspace) return fail(CUBIC_EINVAL, "null workspace");
-    }
+    const int64_t need = launch_workspace(p, m);
+    if (workspace_bytes < need) return fail(CUBIC_EWORKSPACE, "gemm workspace %lld < %lld bytes", (long long)workspace_bytes, (long long)need);
     if (need && !workspace) return fail(CUBIC_EINVAL, "null workspace");
     cubic::GemmArgs a = {};
     a.x = (const uint16_t*)x;
@@ -353,7 +358,7 @@ int gemm_common(const void* x, int64_t ldx, const uint32_t* codes, const uint32_
     a.wide_cols = p.wide_cols;
     a.wide_chunks = p.wide_chunks;
     a.f16 = dtype == CUBIC_DTYPE_F16;
-    if (p.split > 1 && workspace) {
+    if (need) {
         const int64_t counters = align256((int64_t)p.col_blocks * ceil_div(m, p.chunk_rows) * 4);  // one per output block
         a.counters = (uint32_t*)workspace;
         a.partials = (float*)((char*)workspace + counters);
@@ -538,6 +543,18 @@ int64_t cubic_gemm_grouped_workspace_bytes(int64_t m, int64_t n0, int64_t n1, in
     if (n0 == n1) return gemm_workspace_any_group(m, n0, 2, k, bits);
     const int64_t w0 = gemm_workspace_any_group(m, n0, 1, k, bits), w1 = gemm_workspace_any_group(m, n1, 1, k, bits);
     return w0 > w1 ? w0 : w1;
+}
+
+int64_t cubic_gemm_launch_plan(int64_t m, int members, int64_t n, int64_t k, int bits, int group_in, int64_t ldx,
+                               int* kernel, int* split) {
+    if (m <= 0 || n <= 0 || k <= 0 || bits < 1 || bits > 8 || members < 1 || members > cubic::kMaxGemmMembers ||
+        group_in <= 0 || group_in % 32)
+        return -1;
+    const GemmPlan p = plan_launch(m, n, members, k, bits, group_in, ldx);
+    if (kernel)
+        *kernel = p.rows_waves ? CUBIC_GEMM_ROWS : p.panel ? CUBIC_GEMM_PANEL : p.wide_chunks ? CUBIC_GEMM_WIDE : CUBIC_GEMM_TILES;
+    if (split) *split = p.split;
+    return launch_workspace(p, m);
 }
 
 int cubic_gemm(const void* x, int64_t ldx, const uint32_t* codes, const uint32_t* meta,

@@ -114,17 +114,21 @@ def _storage(t: Tensor) -> int:
     return t.untyped_storage().data_ptr()
 
 
-def gemm_workspace_bytes(m: int, widths: Sequence[int], k: int, bits: int) -> int:
-    """Split-K workspace of one bound launch over members of the given widths."""
+def _launch_workspace_bytes(m: int, widths: Sequence[int], k: int, bits: int, group_in: int, ldx: int) -> int:
+    """Workspace that one launch with activation row stride ``ldx`` requires."""
     lib = _native.lib()
     widths = tuple(widths)
-    if len(widths) == 1:
-        return lib.cubic_gemm_workspace_bytes(m, widths[0], k, bits)
     if len(set(widths)) == 1:
-        return lib.cubic_gemm_group_workspace_bytes(m, len(widths), widths[0], k, bits)
-    if len(widths) == 2:
-        return lib.cubic_gemm_grouped_workspace_bytes(m, widths[0], widths[1], k, bits)
+        return lib.cubic_gemm_launch_plan(m, len(widths), widths[0], k, bits, group_in, ldx, None, None)
+    if len(widths) == 2:  # one launch per member
+        return max(lib.cubic_gemm_launch_plan(m, 1, n, k, bits, group_in, ldx, None, None) for n in widths)
     raise ValueError("grouped members of different widths are limited to two")
+
+
+def gemm_workspace_bytes(m: int, widths: Sequence[int], k: int, bits: int) -> int:
+    """Split-K workspace of one bound launch over members of the given widths,
+    whatever its group width: for this m alone (a larger m may need none)."""
+    return max(_launch_workspace_bytes(m, widths, k, bits, group_in, k) for group_in in (128, 32))
 
 
 class _GemmLaunch:
@@ -369,7 +373,8 @@ class PackedLinearOperators:
             raise RuntimeError("Cubic linears must be bound before graph capture")
         prepared = self.prepared(weights, x.device, x.dtype)
         widths = [w.shape[0] for w in weights]
-        ws_bytes = gemm_workspace_bytes(x.shape[0], widths, prepared.k, prepared.bits)
+        ws_bytes = _launch_workspace_bytes(x.shape[0], widths, prepared.k, prepared.bits,
+                                           prepared.group_in, x.stride(0))
         if ws_bytes < 0:
             raise ValueError("invalid GEMM geometry")
         workspace = torch.zeros(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
@@ -448,7 +453,7 @@ def bind_prepared(x: Tensor, prepared: PreparedCubic, outputs: Sequence[Tensor],
     for y, w in zip(outputs, widths):
         if y.shape != (x.shape[0], w) or y.dtype is not prepared.dtype or not y.is_contiguous():
             raise ValueError("bound linear output has an invalid ABI")
-    ws_bytes = gemm_workspace_bytes(x.shape[0], widths, prepared.k, prepared.bits)
+    ws_bytes = _launch_workspace_bytes(x.shape[0], widths, prepared.k, prepared.bits, prepared.group_in, x.stride(0))
     if ws_bytes < 0:
         raise ValueError("invalid GEMM geometry")
     workspace = torch.zeros(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes > 0 else None

@@ -102,11 +102,19 @@ CUBIC_API int cubic_prepare_weight(int fmt, const void* packed, const void* m0, 
  * several tiles, the rest one tile per wave; both issue the same MFMA
  * sequence and agree bit for bit).
  *
- * cubic_gemm_workspace_bytes: workspace for (m, n, k); 0 when no K split.
+ * cubic_gemm_workspace_bytes: workspace for (m, n, k) at any group width and
+ *   row stride; 0 when no K split.  It covers every smaller m as well, so one
+ *   workspace sized at a matrix's largest m serves them all.
  *   The workspace must be zero-filled before its first use; every completed
  *   launch leaves it zero again (a launch killed mid-kernel can leave an
  *   arrival counter set: zero the workspace again before reusing it).  One
  *   workspace per concurrently running launch.
+ * cubic_gemm_launch_plan: what one launch with activation row stride ldx
+ *   takes: returns the workspace that launch itself requires (never more than
+ *   the query above: 0 where it keeps its K partitions in registers; -1 for an
+ *   inadmissible argument) and stores, where the pointers are not NULL, its
+ *   kernel (CUBIC_GEMM_*) and its number of K partitions.  A caller that binds
+ *   one launch at a fixed m may allocate just this.
  * cubic_gemm: single output y[m, ldy] (columns n).
  * cubic_gemm_group: `members` (1..8) matrices of the same [n, k] shape and
  *   encoding sharing x, prepared as one [members * n, k] matrix (member i's
@@ -127,6 +135,12 @@ CUBIC_API int64_t cubic_gemm_group_workspace_bytes(int64_t m, int members, int64
                                                    int bits);
 CUBIC_API int64_t cubic_gemm_grouped_workspace_bytes(int64_t m, int64_t n0, int64_t n1, int64_t k,
                                                      int bits);
+#define CUBIC_GEMM_ROWS 0   /* small rows */
+#define CUBIC_GEMM_PANEL 1  /* column panels */
+#define CUBIC_GEMM_TILES 2  /* MFMA tiles */
+#define CUBIC_GEMM_WIDE 3   /* 256 x 128 tiles */
+CUBIC_API int64_t cubic_gemm_launch_plan(int64_t m, int members, int64_t n, int64_t k, int bits,
+                                         int group_in, int64_t ldx, int* kernel, int* split);
 CUBIC_API int cubic_gemm(const void* x, int64_t ldx, const uint32_t* codes, const uint32_t* meta,
                int64_t m, int64_t n, int64_t k, int bits, int group_in, int dtype, void* y, int64_t ldy,
                void* workspace, int64_t workspace_bytes, void* stream);

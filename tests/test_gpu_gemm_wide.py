@@ -15,6 +15,7 @@ import pytest
 import torch
 
 from cubic_serve_amd import linear, quantization as qz
+from test_gemm_plan_host import TILES, WIDE, launch_plan
 from test_gpu_gemm import random_matrix
 
 pytestmark = pytest.mark.gpu
@@ -66,3 +67,29 @@ def test_wide_is_chosen_where_the_sizes_say():
         assert linear.gemm_workspace_bytes(m, (n,), k, 4) == 0, (n, k, m)
     # 128 wide tiles for 256 CUs and K partitions to use the rest
     assert linear.gemm_workspace_bytes(1024, (4096,), 12288, 4) > 0
+
+
+def test_row_stride_past_the_wide_kernel_equals_contiguous_rows():
+    """A row stride of 2^28 elements, past the wide kernel's offsets: the
+    binding holds the MFMA-tile kernel's K partitions, and the rows equal the
+    contiguous launch bit for bit."""
+    n, members, k, m, stride = 6144, 2, 2048, 129, 1 << 28
+    extent = ((m - 1) * stride + k) * 2
+    if torch.cuda.mem_get_info()[0] < extent + (4 << 30):
+        pytest.skip(f"needs {extent >> 30} GiB of free device memory")
+    print(f"row stride {stride} m={m}", flush=True)
+    assert launch_plan(m, members, n, k, 4, 128)[1] == WIDE
+    need, kernel, split = launch_plan(m, members, n, k, 4, 128, stride)
+    assert kernel == TILES and split > 1 and need > 0
+    parts = [linear.prepare_matrix(random_matrix(n, k, 4, 128, qz.FMT_F32, seed=i).to(DEV), DEV) for i in range(members)]
+    prepared = linear.PreparedCubic(torch.cat([p.codes for p in parts]), torch.cat([p.meta for p in parts]),
+                                    n * members, k, 4, 128, torch.bfloat16)
+    x = torch.randn((m, k), generator=torch.Generator(device=DEV).manual_seed(1), device=DEV).to(torch.bfloat16)
+    far = torch.empty(extent // 2, dtype=torch.bfloat16, device=DEV).as_strided((m, k), (stride, 1))
+    far.copy_(x)
+    got = []
+    for rows in (x, far):
+        ys = [torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(members)]
+        linear.bind_prepared(rows, prepared, ys, (n,) * members).launch()
+        got.append(torch.stack(ys).view(torch.int16))
+    assert torch.equal(got[0], got[1])
