@@ -66,8 +66,6 @@ struct GemmPlan {
 
 #ifdef CUBIC_EXPERIMENTS
 // experiment builds only: force the panel plan (J, split, tables in LDS)
-static int g_wide = 0;  // 1: wide kernel, -1: never
-extern "C" __attribute__((visibility("default"))) void cubic_exp_wide(int w, int) { g_wide = w; }
 static int g_exp_j = 0, g_exp_split = 0, g_exp_tl = -1, g_exp_panel = -1, g_exp_stages = 0, g_exp_waves = 0;
 extern "C" __attribute__((visibility("default"))) void cubic_exp_plan(int j, int split, int tl, int panel, int stages, int waves) {
     g_exp_j = j; g_exp_split = split; g_exp_tl = tl; g_exp_panel = panel; g_exp_stages = stages; g_exp_waves = waves;
@@ -153,41 +151,54 @@ void plan_tiles_per_wave(int64_t m, int group_in, GemmPlan* p) {
 }
 
 // Wide kernel (cubic_wide.hip) instead of the MFMA-tile plan in *p, by the time
-// either is expected to take (us), fitted to launches of M = 200 to 2048 over
-// 2048, 4096 and 8192-wide layers at 4 bits (within about 10% of them):
-//   wide: rounds of 256 workgroups (one per CU), 2.0 per k-block;
-//   MFMA tiles: rounds of 512 workgroups, 2.3 per k-block (two tiles per wave;
-//     64-row chunks, for groups below a k-block, 1.7, and 0.85 with one tile),
-//     a last round of up to 128 workgroups at half, up to 5 a round where
-//     partitions are too short to hide their first loads, and the K split's
-//     partials, written and read at 6.7 TB/s (of two only one is stored).
+// either is expected to take (us):
+//   wide: rounds of 256 workgroups (one per CU), 1.92 per k-block (0.03 less
+//     per bit below 4, 0.19 more with groups below a k-block) and 4.7 to start
+//     and store a tile; a part-filled last round runs its k-blocks up to 0.6
+//     faster;
+//   MFMA tiles: 512 workgroups at a time, 1.89 per k-block (64-row chunks, for
+//     groups below a k-block: 1.28, and 0.75 with one tile per wave, and what
+//     more than two level tables a k-block cost to load; 4.5% less per bit
+//     below 4) and 5.3, 1.7 or 1.6 to start and store; a last round costs more
+//     than its share of 512; and the K split's partials, written and read at
+//     10 TB/s (of two only one is stored).
+// Fitted to 4079 launches of M = 65 to 2300, n 1024 to 151936, k 128 to 28672,
+// bits 1 to 4 and groups of 32 to 256, and checked on 949 others: where the two
+// kernels are within 1.5 times of each other the times are 5 and 7% off (rms);
+// 1.2% of the 949 choices are more than 5% (at most 13%) slower than the other
+// kernel's launch.  (A model without the cost of a tile's start and of the last
+// round's share: 7.5% and 55%.)
 // The wide kernel wins where its 256 x 128 tiles fill their rounds (us, MFMA
-// tiles against wide: 4096 -> 2 x 12288 M = 256 78 / 64, 1024 247 / 206, 2048
-// 487 / 408; 4096 -> 6144 M = 1024 89 / 64; 12288 -> 4096 M = 2048 282 / 195;
-// 2048 -> 2 x 6144 M = 512 65 / 39) and loses where they leave CUs idle that
-// K partitions would use (12288 -> 4096 M = 1024, 128 workgroups, 149 / 164;
-// M = 512 88 / 163; 4096 -> 6144 M = 512 53 / 60).
-void plan_wide(int64_t m, int bits, GemmPlan* p) {
+// tiles / wide: 4096 -> 2 x 12288 M = 256 73 / 61, 1024 245 / 218, 2048 478 /
+// 432; 4096 -> 6144 M = 1024 87 / 63; 12288 -> 4096 M = 2048 272 / 207; 2048 ->
+// 2 x 6144 M = 512 65 / 37) and loses where they leave CUs idle that K
+// partitions would use (12288 -> 4096 M = 1024 149 / 176, M = 512 87 / 162), on
+// a K too short for its start (1024 -> 32768 M = 777 80 / 87, 768 -> 1616 in
+// groups of 64 M = 560 12 / 20) and on a part-filled round over a long K
+// (8192 -> 10240 M = 2048 366 / 388, 8192 -> 2 x 28672 M = 777 885 / 935).
+void plan_wide(int64_t m, int bits, int group_in, GemmPlan* p) {
     // one tile per wave over 128-row chunks: fewer than 320 workgroups of two,
     // never enough for wide tiles
     if (bits > 4 || m <= 64 || (p->chunk_rows == 128 && p->tiles_per_wave == 1)) return;
     const int64_t cols = ceil_div((int64_t)p->n_tiles * 16, cubic::kWideCols);
     const int64_t chunks = ceil_div(m, cubic::kWideRows);
     if (cols * chunks >= (int64_t(1) << 31)) return;
-    const double wide = 2.0 + (double)ceil_div(cols * chunks, 256) * p->k_blocks * 2.0;
+    const int form = p->chunk_rows == 128 ? 0 : p->tiles_per_wave == 2 ? 1 : 2;
+    const double kb = 1.92 - 0.03 * (4 - bits) + (form ? 0.19 : 0.0);
+    const double part = (double)(cols * chunks % 256) / 256;
+    double wide = 6.0 + (double)(cols * chunks / 256) * (p->k_blocks * kb + 4.7);
+    if (part > 0) wide += p->k_blocks * (kb - 0.6 * (1 - part)) + 4.7;
+    constexpr double kStep[3] = {1.89, 1.28, 0.75}, kTable[3] = {0.0, 0.032, 0.016}, kStart[3] = {5.3, 1.7, 1.6};
+    const double tables = (std::max(1.0, (double)kKBlock / group_in) - 2) * (bits == 4 ? 2 : 1);  // past two a k-block
+    const double step = kStep[form] * (1 - 0.045 * (4 - bits)) + kTable[form] * tables;
     const int64_t blocks = (int64_t)p->col_blocks * ceil_div(m, p->chunk_rows);
     const int64_t wgs = blocks * p->split, rest = wgs % 512;
-    const double rounds = (double)(wgs / 512) + (rest == 0 ? 0.0 : rest <= 128 ? 0.5 : 1.0);
-    const double step = p->chunk_rows == 128 ? 2.3 : p->tiles_per_wave == 2 ? 1.7 : 0.85;
-    const double start = p->split > 1 && p->blocks_per_split < 7 ? 7.0 - p->blocks_per_split : 0.0;
+    double rounds = (double)(wgs / 512);
+    if (rest) rounds += std::min(1.0, 0.45 + 0.7 * (double)rest / 512);
     const double stored = p->split == 1 ? 0.0 : p->split == 2 ? 1.0 : (double)p->split;
     const double block_bytes = 8.0 * p->chunk_rows * (16 * cubic::kGemmWaves * p->tiles_per_wave);
-    const double tiles = rounds * (p->blocks_per_split * step + start) + stored * (double)blocks * block_bytes / 6.7e6;
-    bool take = wide < tiles;
-#ifdef CUBIC_EXPERIMENTS
-    if (g_wide) take = g_wide > 0;
-#endif
-    if (!take) return;
+    const double tiles = 8.0 + rounds * (p->blocks_per_split * step + kStart[form]) + stored * (double)blocks * block_bytes / 10e6;
+    if (wide >= tiles) return;
     p->wide_cols = (int)cols;
     p->wide_chunks = (int)chunks;
 }
@@ -247,7 +258,7 @@ GemmPlan plan_gemm(int64_t m, int64_t n_member, int members, int64_t k, int bits
         }
     }
     plan_tiles_per_wave(m, group_in, &p);
-    plan_wide(m, bits, &p);
+    plan_wide(m, bits, group_in, &p);
     return p;
 }
 

@@ -73,3 +73,31 @@ def test_bound_launches_allocate_what_they_need():
     assert launch_plan(64, 9, 6144, 4096, 4, 128)[0] == -1
     assert launch_plan(64, 1, 6144, 4096, 9, 128)[0] == -1
     assert launch_plan(64, 1, 6144, 4096, 4, 100)[0] == -1
+
+
+# n per member, members, k, bits, group, m, us on the MFMA-tile kernel, us on the wide kernel
+MEASURED = [
+    (1616, 1, 768, 2, 64, 560, 12.2, 19.9), (3224, 1, 768, 2, 64, 281, 12.8, 19.5),
+    (18768, 1, 1024, 1, 64, 899, 50.5, 66.2), (21480, 1, 2272, 4, 32, 428, 69.1, 83.1),
+    (32768, 1, 1024, 4, 128, 384, 39.6, 44.2), (32768, 1, 1024, 4, 128, 777, 80.3, 87.2),
+    (34928, 1, 2816, 4, 32, 246, 86.9, 98.7), (20248, 1, 1248, 2, 32, 1055, 84.4, 97.2),
+    (10240, 1, 8192, 4, 128, 2048, 365.6, 388.2), (28672, 2, 8192, 4, 128, 777, 885.0, 935.5),
+    (29152, 1, 6912, 4, 128, 1288, 630.5, 670.6), (34224, 1, 12736, 4, 128, 2055, 1844.4, 1992.1),
+    (14896, 1, 20224, 4, 256, 2135, 1421.7, 1514.2),
+    (4096, 1, 12288, 4, 128, 1024, 148.1, 176.0), (4096, 1, 12288, 4, 128, 512, 86.8, 162.1),
+    (12288, 2, 4096, 4, 128, 300, 101.9, 121.7), (6144, 1, 4096, 4, 128, 384, 45.0, 59.4),
+    (12288, 2, 4096, 4, 128, 256, 72.8, 61.4), (12288, 2, 4096, 4, 128, 2048, 478.1, 433.0),
+    (6144, 1, 4096, 4, 128, 1024, 87.5, 62.7), (4096, 1, 12288, 4, 128, 2048, 272.4, 206.4),
+    (6144, 2, 2048, 4, 128, 512, 64.8, 36.5), (3072, 1, 3072, 4, 128, 2048, 136.8, 53.5),
+    (4096, 1, 4096, 3, 128, 1536, 87.0, 62.3), (12288, 2, 4096, 4, 32, 777, 298.5, 231.7),
+    (12288, 2, 4096, 2, 32, 512, 168.4, 135.7), (32768, 1, 128, 4, 128, 2048, 85.8, 75.0),
+    (151936, 1, 4096, 4, 32, 200, 468.5, 371.4),
+]
+
+
+@pytest.mark.parametrize("n,members,k,bits,group,m,tiles,wide", MEASURED)
+def test_plan_takes_the_kernel_that_measured_faster(n, members, k, bits, group, m, tiles, wide):
+    """Both kernels' times on an MI355X, 4 to 160% apart: the first thirteen
+    were planned wide by a model without a tile's start and the last round's
+    share."""
+    assert launch_plan(m, members, n, k, bits, group)[1] == (WIDE if wide < tiles else TILES)
