@@ -196,6 +196,7 @@ class CapturedGreedySampler:
                  graph_pool=None, consume_logits: bool = False) -> None:
         dev = token_ids.device
         self.device = dev
+        self._index = dev.index  # device guards and stream lookups take the integer faster
         self.capacity = token_ids.numel()
         if (dev.type != "cuda" or token_ids.ndim != 1 or self.capacity < 1
                 or type(true_vocab_size) is not int or true_vocab_size < 1):
@@ -240,18 +241,21 @@ class CapturedGreedySampler:
 
     def launch(self) -> None:
         """Enqueue the fused launch on the current stream (metadata as it stands)."""
+        with torch.cuda.device(self._index):
+            self._enqueue()
+
+    def _enqueue(self) -> None:
         w, p = self.workspace, self.parameters
-        with torch.cuda.device(self.device):
-            _native.call("cubic_greedy_sample", self.logits.data_ptr(),
-                         int(self.logits.dtype == torch.float16), self.logits.stride(0),
-                         self.capacity, self.width, self.metadata.data_ptr(),
-                         _native.ptr(self.token_mask), self._mask_words,
-                         _native.ptr(self.masked_logits), self._masked_stride, p.max_top_k,
-                         *_param_ptrs(p), self.vocab_size, w.local_scores.data_ptr(),
-                         w.local_token_ids.data_ptr(), self.token_ids.data_ptr(),
-                         self.root_valid.data_ptr(), self.final_valid.data_ptr(),
-                         self._scratch.data_ptr(), self._scratch.numel(),
-                         _native.stream_of(self.device))
+        _native.call("cubic_greedy_sample", self.logits.data_ptr(),
+                     int(self.logits.dtype == torch.float16), self.logits.stride(0),
+                     self.capacity, self.width, self.metadata.data_ptr(),
+                     _native.ptr(self.token_mask), self._mask_words,
+                     _native.ptr(self.masked_logits), self._masked_stride, p.max_top_k,
+                     *_param_ptrs(p), self.vocab_size, w.local_scores.data_ptr(),
+                     w.local_token_ids.data_ptr(), self.token_ids.data_ptr(),
+                     self.root_valid.data_ptr(), self.final_valid.data_ptr(),
+                     self._scratch.data_ptr(), self._scratch.numel(),
+                     _native.stream_of(self._index))
 
     def _set_metadata(self, count: int, cancel: bool) -> None:
         if type(count) is not int or not 0 < count <= self.capacity or type(cancel) is not bool:
@@ -270,11 +274,16 @@ class CapturedGreedySampler:
             raise TensorParallelSamplingError("greedy graph replay is unavailable")
         if validity_out is not None:
             _require(validity_out, (), torch.bool, self.device, "deferred sampling validity")
-        self._set_metadata(count, cancel)
-        # the graph holds this one launch: enqueueing it directly costs the
-        # host 6 us where a graph launch costs 16 (64 rows x 151936: 25 -> 15
-        # us a call, of which the kernel is 10)
-        self.launch()
+        with torch.cuda.device(self._index):
+            # a capture would hold the launch but not (or only at its own
+            # replay) the metadata write that this object counts as done
+            if torch.cuda.is_current_stream_capturing():
+                raise TensorParallelSamplingError("greedy graph replay is unavailable under stream capture")
+            self._set_metadata(count, cancel)
+            # the graph holds this one launch: enqueueing it directly costs the
+            # host 6 us where a graph launch costs 16 (64 rows x 151936: 25 -> 15
+            # us a call, of which the kernel is 10)
+            self._enqueue()
         if validity_out is not None:
             validity_out.copy_(self.final_valid)
             return self.token_ids

@@ -291,6 +291,46 @@ def test_captured_sampler_reference_corpus(oracle, dtype):
     assert side.item() > 0
 
 
+def make_sampler(capacity, width, dtype=torch.bfloat16):
+    """(sampler, its logits) with parameters every row admits."""
+    logits = torch.zeros((capacity, width), dtype=dtype, device=DEV)
+    ws = ShardedSamplingWorkspace(torch.empty((capacity, 20), dtype=dtype, device=DEV),
+                                  torch.empty((capacity, 20), dtype=torch.int64, device=DEV), None, None)
+    return CapturedGreedySampler(local_logits=logits, true_vocab_size=width,
+                                 token_ids=torch.empty(capacity, dtype=torch.int64, device=DEV),
+                                 parameters=params(capacity), workspace=ws,
+                                 root_valid=torch.empty(capacity, dtype=torch.bool, device=DEV)), logits
+
+
+def test_replay_is_refused_under_capture_and_leaves_the_metadata():
+    """A capture would hold the launch without the (count, cancel) write that
+    the sampler counts as done: replay refuses, whether the pair is new or the
+    one last written, and the next eager replays still write theirs.  launch()
+    is what a capture records: it reads the metadata as it stands."""
+    capacity, width = 4, 300
+    plan, logits = make_sampler(capacity, width)
+    logits.copy_(tie_logits(capacity, width, torch.bfloat16, torch.Generator().manual_seed(4)))
+    valid = torch.zeros((), dtype=torch.bool, device=DEV)
+    want = {n: plan.replay(n).tolist() for n in (1, 2, 3, 4)}
+    assert [w.count(-1) for w in want.values()] == [3, 2, 1, 0]
+    plan.replay(2)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for count in (2, 3):                     # the pair last written, a new one
+            with pytest.raises(TensorParallelSamplingError, match="capture"):
+                plan.replay(count, validity_out=valid)
+        plan.launch()
+    assert plan.replay(3).tolist() == want[3]    # written, not taken for done
+    for count in (1, 4, 2):
+        assert plan.replay(count).tolist() == want[count]
+        plan.token_ids.fill_(77)
+        graph.replay()                           # the count last written, now
+        torch.cuda.synchronize()
+        assert plan.token_ids.tolist() == want[count] and bool(plan.final_valid)
+    graph.reset()
+    plan.close()
+
+
 def _expected_masked(logits_bits, mask, start, active, ninf):
     """local_candidates.cu:37-53: row r < active keeps the admitted columns'
     bits and -inf elsewhere; rows >= active are -inf."""
