@@ -186,7 +186,9 @@ class CapturedGreedySampler:
     ``root_valid``, and the batch validity into ``final_valid``.  ``replay``
     writes the (count, cancel) metadata from a pinned host table, enqueues the
     graph's launch, and raises TensorParallelSamplingError when the batch is
-    rejected.  ``graph`` itself is for callers that replay it inside their own.
+    rejected.  Replays, ``launch`` and ``graph`` (for callers that replay it
+    themselves) share the outputs, the metadata and the scratch counters: the
+    caller orders calls that are on different streams.
     """
 
     def __init__(self, *, local_logits: Tensor, true_vocab_size: int, token_ids: Tensor,

@@ -15,7 +15,9 @@ cubic_sampling_final_guard, cubic_greedy_sample) against the CPU oracle.
 * the fused single-GPU launch equal to the composition of the three, and the
   reference's captured-sampler test (tests/ops/test_cuda_greedy_sampling.py:
   95-190): every count of each capacity, both row orders, invalid parameters
-  rejected, replays of one captured graph interleaved with eager work.
+  rejected, replays (one launch each) interleaved with eager work, and the
+  sampler's captured graph after each of them, for callers that replay it
+  themselves.
 """
 from __future__ import annotations
 
@@ -238,6 +240,23 @@ def test_fused_sample_equals_composition(oracle, dtype, rows, width):
                 np.testing.assert_array_equal(g, w)
 
 
+def check_graph(plan):
+    """The captured graph, at the metadata of the last replay, rewrites every
+    output of that replay."""
+    outputs = (plan.token_ids, plan.root_valid, plan.final_valid, plan.workspace.local_scores,
+               plan.workspace.local_token_ids)
+    if plan.masked_logits is not None:
+        outputs += (plan.masked_logits,)
+    want = [t.clone() for t in outputs]
+    for t, w in zip(outputs, want):
+        t.copy_(~w if w.dtype == torch.bool else torch.full_like(w, 77))
+    plan.graph.replay()
+    torch.cuda.synchronize()
+    for t, w in zip(outputs, want):
+        assert torch.equal(t.view(torch.int16) if t.dtype == plan.logits.dtype else t,
+                           w.view(torch.int16) if w.dtype == plan.logits.dtype else w)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_captured_sampler_reference_corpus(oracle, dtype):
     """tests/ops/test_cuda_greedy_sampling.py:95-190 on one GPU (TP = 1)."""
@@ -272,6 +291,7 @@ def test_captured_sampler_reference_corpus(oracle, dtype):
                     expected = [reference[r] for r in perm] + [-1] * (capacity - count)
                     assert out.cpu().tolist() == expected
                     assert plan.root_valid.cpu().tolist() == [True] * count + [False] * (capacity - count)
+                    check_graph(plan)
             count = min(capacity, 3)
             for buffer, value in ((p.temperatures, 1), (p.top_ps, 0), (p.top_ks, 21), (p.ordinals, -1)):
                 saved = buffer.clone()
@@ -282,10 +302,12 @@ def test_captured_sampler_reference_corpus(oracle, dtype):
             if count < capacity:
                 plan.replay(count, True)                          # cancel: -2 after the last row
                 assert plan.token_ids[count].item() == -2
+                check_graph(plan)
             logits[0, 5] = float("inf")
             with pytest.raises(TensorParallelSamplingError, match="invalid"):
                 plan.replay(count, False)
             assert plan.token_ids[0].item() == -1
+            check_graph(plan)
         finally:
             plan.close()
     assert side.item() > 0
@@ -396,7 +418,8 @@ def test_masked_logits_output_and_consumption(oracle, dtype):
 
 def test_captured_sampler_writes_masked_logits(oracle):
     """CapturedGreedySampler(token_mask=, masked_logits=) (greedy.py:49-69):
-    every replay rewrites the masked logits for the count it runs."""
+    every replay, and the captured graph, rewrites the masked logits for the
+    count it runs."""
     dtype, capacity, width = torch.bfloat16, 4, 3000
     gen = torch.Generator().manual_seed(22)
     logits = tie_logits(capacity, width, dtype, gen)
@@ -417,5 +440,6 @@ def test_captured_sampler_writes_masked_logits(oracle):
             plan.replay(count, False)
             torch.cuda.synchronize()
             np.testing.assert_array_equal(bits(out), _expected_masked(bits(logits), mask, 0, count, 0xFF80))
+            check_graph(plan)
     finally:
         plan.close()
