@@ -152,20 +152,19 @@ void plan_tiles_per_wave(int64_t m, int group_in, GemmPlan* p) {
 
 // Wide kernel (cubic_wide.hip) instead of the MFMA-tile plan in *p, by the time
 // either is expected to take (us):
-//   wide: rounds of 256 workgroups (one per CU), 1.92 per k-block (0.03 less
-//     per bit below 4, 0.19 more with groups below a k-block) and 4.7 to start
-//     and store a tile; a part-filled last round runs its k-blocks up to 0.6
-//     faster;
-//   MFMA tiles: 512 workgroups at a time, 1.89 per k-block (64-row chunks, for
-//     groups below a k-block: 1.28, and 0.75 with one tile per wave, and what
-//     more than two level tables a k-block cost to load; 4.5% less per bit
-//     below 4) and 5.3, 1.7 or 1.6 to start and store; a last round costs more
-//     than its share of 512; and the K split's partials, written and read at
-//     10 TB/s (of two only one is stored).
+//   wide: rounds of 256 workgroups (one per CU), 1.93 per k-block at 4 bits
+//     (0.19 more with groups below a k-block) and 4.7 to start and store a
+//     tile; a part-filled last round runs its k-blocks up to 0.6 faster;
+//   MFMA tiles: 512 workgroups at a time, 1.89 per k-block at 4 bits (64-row
+//     chunks, for groups below a k-block: 1.28, and 0.75 with one tile per
+//     wave, and what more than two level tables a k-block cost to load) and
+//     5.3, 1.7 or 1.6 to start and store; a last round costs more than its
+//     share of 512; and the K split's partials, written and read at 10 TB/s
+//     (of two only one is stored).
 // Fitted to 4079 launches of M = 65 to 2300, n 1024 to 151936, k 128 to 28672,
 // bits 1 to 4 and groups of 32 to 256, and checked on 949 others: where the two
 // kernels are within 1.5 times of each other the times are 5 and 7% off (rms);
-// 1.2% of the 949 choices are more than 5% (at most 13%) slower than the other
+// 1.4% of the 949 choices are more than 5% (at most 13%) slower than the other
 // kernel's launch.  (A model without the cost of a tile's start and of the last
 // round's share: 7.5% and 55%.)
 // The wide kernel wins where its 256 x 128 tiles fill their rounds (us, MFMA
@@ -184,13 +183,14 @@ void plan_wide(int64_t m, int bits, int group_in, GemmPlan* p) {
     const int64_t chunks = ceil_div(m, cubic::kWideRows);
     if (cols * chunks >= (int64_t(1) << 31)) return;
     const int form = p->chunk_rows == 128 ? 0 : p->tiles_per_wave == 2 ? 1 : 2;
-    const double kb = 1.92 - 0.03 * (4 - bits) + (form ? 0.19 : 0.0);
+    constexpr double kWide[4] = {1.83, 1.87, 1.82, 1.93}, kTiles[4] = {0.87, 0.96, 0.95, 1.0};  // by bits
+    const double kb = kWide[bits - 1] + (form ? 0.19 : 0.0);
     const double part = (double)(cols * chunks % 256) / 256;
     double wide = 6.0 + (double)(cols * chunks / 256) * (p->k_blocks * kb + 4.7);
     if (part > 0) wide += p->k_blocks * (kb - 0.6 * (1 - part)) + 4.7;
     constexpr double kStep[3] = {1.89, 1.28, 0.75}, kTable[3] = {0.0, 0.032, 0.016}, kStart[3] = {5.3, 1.7, 1.6};
     const double tables = (std::max(1.0, (double)kKBlock / group_in) - 2) * (bits == 4 ? 2 : 1);  // past two a k-block
-    const double step = kStep[form] * (1 - 0.045 * (4 - bits)) + kTable[form] * tables;
+    const double step = kStep[form] * kTiles[bits - 1] + kTable[form] * tables;
     const int64_t blocks = (int64_t)p->col_blocks * ceil_div(m, p->chunk_rows);
     const int64_t wgs = blocks * p->split, rest = wgs % 512;
     double rounds = (double)(wgs / 512);
