@@ -1,8 +1,9 @@
 // Device helpers shared by the Cubic GEMM kernels (cubic_gemm.hip,
-// cubic_panel.hip): the activation LDS swizzle, the level-table decode, the
-// prepared-code loads and the output / split-K epilogue.  Every kernel that
-// uses them performs the same per-tile arithmetic, so their outputs agree bit
-// for bit under one K plan.
+// cubic_panel.hip, cubic_wide.hip): the activation LDS swizzle, the level-table
+// decode, the prepared-code loads and the output / split-K epilogue.  Every
+// kernel that uses them performs the same per-tile arithmetic, so their outputs
+// agree bit for bit under one K plan.  (The wide kernel has its own activation
+// layout and epilogue.)
 #pragma once
 #include "cubic_device.h"
 #include "cubic_capi_internal.h"
@@ -22,14 +23,14 @@ constexpr int kKBlock = 128;
 // (lanes 0..15 store rows 0..15 of one chunk) in position r ^ g(c): both run at
 // the b128 peak rate of gfx950's LDS (measured 243 B/clk/CU for the reads,
 // 83 B/clk/CU for the writes; the plain r ^ c swizzle reads at 128).
+__device__ __forceinline__ int a_slot(int r16, int c) { return c * 16 + (r16 ^ ((c & 3) << 2) ^ (c >> 2)); }
 // bf16 per activation stage of a workgroup with MT m-tiles (the output tile
 // of the epilogue fits two stages at every MT).  Stages of 64 rows whatever
 // MT held 32 KB of LDS for 8 KB of activations and set the workgroups per CU
-// of wide launches at M <= 16 and above 4 bits: Llama-3-70B gate/up at M = 8
-// 138 -> 128 us at 6 bits, 161 -> 147 at 8.
+// at M <= 16 above 4 bits (M = 8, us): 8192 -> 2 x 28672 at 6 bits 126 -> 118,
+// at 8 bits 143 -> 130; 28672 -> 8192 at 7 bits 96 -> 75; 8192 -> 10240 within 2%.
 template <int MT>
 __host__ __device__ constexpr int a_stage() { return MT * 16 * kKBlock; }
-__device__ __forceinline__ int a_slot(int r16, int c) { return c * 16 + (r16 ^ ((c & 3) << 2) ^ (c >> 2)); }
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float floatx4_t;
@@ -165,8 +166,9 @@ __device__ __forceinline__ uint32_t code_at(const uint32_t* w, int i) {
 
 // Signs of the pair of codes 2 p, 2 p + 1 of a lane's words in bits 15 and 31,
 // both at once: two or three VALU a pair where one by one it is six, and VALU
-// bounds the decode of these widths.  8 bits, M = 8, 28672 x 2 x 8192 147 ->
-// 137 us, 10240 x 8192 38.6 -> 36.6; M = 64 204 -> 188.
+// bounds the decode of these widths.  8 bits (us): 8192 -> 2 x 28672 M = 8 138
+// -> 130, M = 64 190 -> 180; 8192 -> 10240 37.3 -> 35.3 and 45.3 -> 43.4; 12288
+// -> 4096, fp16, M = 333 115 -> 111.  6 and 7 bits within 3%.
 template <int BITS>
 __device__ __forceinline__ uint32_t pair_signs(const uint32_t* w, int p, uint32_t c0, uint32_t c1) {
     if constexpr (BITS == 8)  // the codes are bytes: into bytes 1 and 3 (selector 4: a zero byte)

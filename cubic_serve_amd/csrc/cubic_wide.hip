@@ -4,7 +4,8 @@
 // Same prepared weights and the same per-tile arithmetic as gemm_kernel: per
 // (m-tile, tile, k-block, fragment) one v_mfma_f32_16x16x32 in the same order,
 // every K partition of the plan summed from zero and the partitions added in
-// ascending order, so a row's output is the same bits at every M.
+// ascending order, so a row's output is the same bits at every M >= 5 (and
+// below where the small-row kernel, with partitions of its own, does not run).
 //
 // What bounds it: the matrix cores, if the rest hides under them.  gemm_kernel
 // decodes each weight M / 128 times, feeds two MFMAs per A fragment read from
@@ -24,8 +25,9 @@
 //  - K partitions are folded in registers (`tot`), so K is never split over
 //    workgroups and no FP32 partial reaches memory.
 // Measured at M = 2048, W4 g128 (us, gemm_kernel -> this; a plain bf16 library
-// product of the decoded matrix): 4096 -> 6144 171 -> 127, 4096 -> 4096 116 ->
-// 71 (61), 4096 -> 2 x 12288 495 -> 408 (330), 12288 -> 4096 283 -> 195 (180).
+// product of the decoded matrix): 4096 -> 6144 161 -> 135 (89), 4096 -> 4096
+// 107 -> 67 (57), 4096 -> 2 x 12288 463 -> 420 (279), 12288 -> 4096 268 -> 201
+// (180).
 // Time per k-block and round of 256 workgroups: 2.0 us, of which the MFMAs
 // alone take 1.1; the DMA's and the LDS reads' latency inside the halves is
 // the rest (without the DMA 1.8, without the code loads 1.9).

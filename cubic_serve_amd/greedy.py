@@ -283,7 +283,7 @@ class CapturedGreedySampler:
                 raise TensorParallelSamplingError("greedy graph replay is unavailable under stream capture")
             self._set_metadata(count, cancel)
             # the graph holds this one launch: enqueueing it directly costs the
-            # host 6 us where a graph launch costs 16 (64 rows x 151936: 25 -> 15
+            # host 6 us where a graph launch costs 16 (64 rows x 151936: 25 -> 13
             # us a call, of which the kernel is 10)
             self._enqueue()
         if validity_out is not None:

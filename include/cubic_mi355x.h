@@ -97,10 +97,13 @@ CUBIC_API int cubic_prepare_weight(int fmt, const void* packed, const void* m0, 
  * The regimes, as the reference's: m <= 4 with groups of whole 128-wide
  * k-blocks runs the small-row kernel (bits <= 4 at any k; 5..8 bits while k
  * is at most 64 k-blocks), one partition per wave, a function of k alone;
- * every other m runs the MFMA-tile arithmetic with the K plan above (m <= 64
+ * every other m runs the MFMA-tile arithmetic with the K plan above: m <= 64
  * at bits <= 4 on column panels that share each staged activation block over
- * several tiles, the rest one tile per wave; both issue the same MFMA
- * sequence and agree bit for bit).
+ * several tiles, prompt-sized m at bits <= 4 on 256 x 128 tiles that decode
+ * each weight once and add the K partitions in registers where that is
+ * expected to be faster, the rest on one or two tiles per wave.  All three
+ * issue the same MFMA sequence, add the partitions in the same order and agree
+ * bit for bit.
  *
  * cubic_gemm_workspace_bytes: workspace for (m, n, k) at any group width and
  *   row stride; 0 when no K split.  It covers every smaller m as well, so one
